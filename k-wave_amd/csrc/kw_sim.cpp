@@ -812,11 +812,15 @@ void ckpt_header(const kw_sim* s, uint64_t* h) {
 // grid shape and physics branch for the process (the serving loop tunes each
 // shape once).
 namespace {
+// kinds: which specialised kernels the handle has.  A configuration found with
+// some of them switched off (by the environment, or replaced by the radial pass)
+// names sizes that a handle with them must not take: generic kernels on padded
+// spectrum rows, or narrow tiles where the generic last axis was asked for.
 struct TuneKey {
-  int Nx, Ny, Nz, kxm, absorbing, nonlinear, psrc, usrc;
+  int Nx, Ny, Nz, kxm, absorbing, nonlinear, psrc, usrc, kinds;
   bool operator<(const TuneKey& o) const {
-    return std::tie(Nx, Ny, Nz, kxm, absorbing, nonlinear, psrc, usrc) <
-           std::tie(o.Nx, o.Ny, o.Nz, o.kxm, o.absorbing, o.nonlinear, o.psrc, o.usrc);
+    return std::tie(Nx, Ny, Nz, kxm, absorbing, nonlinear, psrc, usrc, kinds) <
+           std::tie(o.Nx, o.Ny, o.Nz, o.kxm, o.absorbing, o.nonlinear, o.psrc, o.usrc, o.kinds);
   }
 };
 struct TuneCfg {
@@ -835,8 +839,10 @@ std::mutex g_tune_mu;
 std::map<TuneKey, std::shared_ptr<TuneEntry>> g_tune_cache;
 
 TuneKey tune_key(const kw_sim* s) {
+  const int kinds = (s->xl.nt ? 1 : 0) | (s->tly.nt ? 2 : 0) | (s->tll.nt ? 4 : 0) | (s->xl.len ? 8 : 0) |
+                    (s->tly.len ? 16 : 0) | (s->tll.len ? 32 : 0) | (s->axisym ? 64 : 0);
   return TuneKey{s->g.Nx,        s->g.Ny, s->g.Nz, s->g.kxm, s->m.absorbing, s->m.nonlinear,
-                 (int)(s->psrc.flag > 0), (int)(s->usrc[0].flag + s->usrc[1].flag + s->usrc[2].flag > 0)};
+                 (int)(s->psrc.flag > 0), (int)(s->usrc[0].flag + s->usrc[1].flag + s->usrc[2].flag > 0), kinds};
 }
 
 void apply_cfg(kw_sim* s, const TuneCfg& c) {
