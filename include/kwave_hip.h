@@ -207,9 +207,11 @@ kw_status kw_sim_autotune(kw_sim* sim, int trial_steps, int* row_nt, int* pencil
 
 /* The launch configuration a handle runs with (after kw_sim_autotune, the
  * tuned one): workgroup sizes of the x-row kernels, the y pass, the
- * last-axis pass and the plane pass (0: kind not used by this grid), and the
- * radix plans of the two pencil passes (0: radices 16, 8, 4, 2, 3, 5, 7
- * greedily; 1: radix 8 at most).  No counterpart in the reference. */
+ * last-axis pass and the plane pass (0: kind not used by this grid, or run by
+ * the generic kernels), and the radix plans of the two pencil passes (0: radices
+ * 16, 8, 4, 2, 3, 5, 7 greedily; 1: radix 8 at most; 4: the fewest stages with
+ * radices up to 10, the plan of the lengths that have one instantiation).  No
+ * counterpart in the reference. */
 typedef struct kw_launch_config {
   int32_t row_nt, ypass_nt, last_nt, plane_nt;
   int32_t ypass_plan, last_plan;

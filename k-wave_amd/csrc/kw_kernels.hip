@@ -793,10 +793,10 @@ const LenKernels* len_kernels(int n) {
   ((nt) == 64 ? fn<64>(__VA_ARGS__)                             \
               : (nt) == 128 ? fn<128>(__VA_ARGS__) : (nt) == 256 ? fn<256>(__VA_ARGS__) : false)
 
-// pencils: 128 to 1024 threads (64 in the environment runs the 128-thread form)
+// pencils: 128 to 1024 threads
 #define KW_BY_NT_PENCIL(nt, fn, ...)                                                   \
   ((nt) == 1024 ? fn<1024>(__VA_ARGS__) : (nt) == 512 ? fn<512>(__VA_ARGS__)           \
-   : (nt) == 256 ? fn<256>(__VA_ARGS__) : (nt) != 0 ? fn<128>(__VA_ARGS__) : false)
+   : (nt) == 256 ? fn<256>(__VA_ARGS__) : (nt) == 128 ? fn<128>(__VA_ARGS__) : false)
 
 static bool ypass_fast(hipStream_t s, const Grid& g, int n, const float2* tw, float2* const* f, int nf, float sign,
                        int nt, int plan) {

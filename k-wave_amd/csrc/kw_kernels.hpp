@@ -379,6 +379,7 @@ struct LenKernels {
   void (*last)(hipStream_t, const Grid&, const float2* tw, const LastArgs&, const SpecTables&);
   void (*last_narrow)(hipStream_t, const Grid&, const float2* tw, const LastArgs&, const SpecTables&);
   RadialFn radial;  // even lengths 2 Ny of axisymmetric grids, else nullptr
+  int row_nt, y_nt, last_nt;  // workgroup sizes of the x rows, y pass and last axis
 };
 // nullptr: the length is in KW_FAST_SIZES, or only the runtime-radix kernels take it
 const LenKernels* len_kernels(int n);
@@ -393,7 +394,7 @@ struct XLaunch {
 struct TileLaunch {
   int tx;       // pencils per workgroup (generic kernels)
   int threads;
-  int nt;       // workgroup size of the length-specialised kernels (64/128/256/512; 0 = none of them)
+  int nt;       // workgroup size of the length-specialised kernels (128/256/512/1024; 0 = none of them)
   int plan;     // radix plan of the length-specialised kernels (kwt::next_radix; 1 only for lengths >= 160)
   int narrow = 0;  // last axis of 2-D grids: 4-column tiles (launch_last_narrow) instead of nt
   const LenKernels* len = nullptr;  // with nt 0: the length's kernels (nullptr = generic only)

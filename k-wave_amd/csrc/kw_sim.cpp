@@ -290,13 +290,15 @@ TileLaunch choose_tile(int width, int n, int nbuf) {
   return TileLaunch{tx, 256, 0, 0};
 }
 
-// Thread count for the length-specialised kernels: 64, 128 or 256, or 0 to
-// use the generic kernels; an environment variable overrides the default.
-int env_nt(const char* name, int def, bool allow512 = false) {
+// Thread count for the length-specialised kernels: 64, 128 or 256 (pencils: 128
+// to 1024, and 64 runs the 128-thread form), or 0 to use the generic kernels;
+// an environment variable overrides the default.
+int env_nt(const char* name, int def, bool pencil = false) {
   const char* v = std::getenv(name);
   if (!v || !*v) return def;
   const int n = std::atoi(v);
-  return (n == 0 || n == 64 || n == 128 || n == 256 || (allow512 && (n == 512 || n == 1024))) ? n : def;
+  if (pencil && n == 64) return 128;
+  return (n == 0 || n == 64 || n == 128 || n == 256 || (pencil && (n == 512 || n == 1024))) ? n : def;
 }
 
 // Radix plan of a pencil length from the environment (0 or 1; plan 1 is
@@ -1742,8 +1744,10 @@ kw_status kw_sim_autotune(kw_sim* s, int trial_steps, int* row_nt, int* pencil_n
     }
     apply_cfg(s, best);
     reset_state(s);
-    if (row_nt) *row_nt = s->xl.nt;
-    if (pencil_nt) *pencil_nt = s->tly.nt ? s->tly.nt : s->tll.nt;
+    kw_launch_config lc;
+    kw_sim_launch_config(s, &lc);
+    if (row_nt) *row_nt = lc.row_nt;
+    if (pencil_nt) *pencil_nt = lc.ypass_nt ? lc.ypass_nt : lc.last_nt;
     if (plane_nt) *plane_nt = s->plane_nt;
   } catch (const HipError& e) {
     return fail(KW_ERR_DEVICE, "HIP error %d (%s) in %s", (int)e.e, hipGetErrorString(e.e), e.what);
@@ -1753,14 +1757,25 @@ kw_status kw_sim_autotune(kw_sim* s, int trial_steps, int* row_nt, int* pencil_n
 
 kw_status kw_sim_launch_config(const kw_sim* s, kw_launch_config* c) {
   if (!s || !c) return fail(KW_ERR_INVALID, "null argument");
-  c->row_nt = s->xl.nt;
-  c->ypass_nt = s->g.dim == 3 && !s->g.kxm && !s->axisym ? s->tly.nt : 0;
-  c->last_nt = s->g.kxm || s->axisym || !s->tll.nt ? 0 : s->tll.narrow ? narrow_threads(s->axL.n) : s->tll.nt;
-  c->plane_nt = s->g.kxm ? (s->plane_nt ? s->plane_nt : default_plane_nt(s->g.Ny, s->g.Nz)) : 0;
-  c->ypass_plan = c->ypass_nt ? s->tly.plan : 0;
-  c->last_plan = c->last_nt ? s->tll.plan : 0;
+  *c = kw_launch_config{};
+  // a length has the tuned kernels (nt), one instantiation (len, plan 4) or only
+  // the generic ones, in the order in which the launchers try them
+  const XLaunch& x = s->xl;
+  c->row_nt = x.nt ? x.nt : x.len ? x.len->row_nt : 0;
+  c->row_wg_target = c->row_nt ? s->g.row_wgs : 0;
   c->kx_major = s->g.kxm;
-  c->row_wg_target = s->xl.nt ? s->g.row_wgs : 0;
+  if (s->g.kxm) {
+    c->plane_nt = s->plane_nt ? s->plane_nt : default_plane_nt(s->g.Ny, s->g.Nz);
+  } else if (!s->axisym) {
+    const TileLaunch &y = s->tly, &l = s->tll;
+    if (s->g.dim == 3) {
+      c->ypass_nt = y.nt ? y.nt : y.len ? y.len->y_nt : 0;
+      c->ypass_plan = y.nt ? y.plan : y.len ? 4 : 0;
+    }
+    const bool narrow = l.narrow && (l.nt || l.len);
+    c->last_nt = narrow ? narrow_threads(s->axL.n) : l.nt ? l.nt : l.len ? l.len->last_nt : 0;
+    c->last_plan = l.nt ? (narrow ? 0 : l.plan) : l.len ? 4 : 0;
+  }
   return KW_OK;
 }
 
@@ -1843,7 +1858,7 @@ kw_status kw_diag_copy_ex(uint64_t bytes, int device, int variant, int blocks, d
 // takes the wide form (kw_xrow.inc).  Both forms are one body with the same
 // butterflies and update expressions, and multiply-adds fuse within one source
 // expression only (-ffp-contract=on), so results are the same bit for bit
-// (tested on every tuned row length and medium).
+// (tested).
 // =============================================================================
 namespace {
 
