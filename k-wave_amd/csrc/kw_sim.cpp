@@ -14,6 +14,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <tuple>
 #include <utility>
 #include <string>
@@ -1716,22 +1717,28 @@ kw_status kw_sim_autotune(kw_sim* s, int trial_steps, int* row_nt, int* pencil_n
           trial(c);
         }
       }
-      // (axisymmetric grids: the radial pass replaces the pencils)
+      // (axisymmetric grids: the radial pass replaces the pencils).  An axis without
+      // tuned kernels keeps its one launch shape: the pairs that differ only there
+      // are the same launch, and are timed once
       if (!s->g.kxm && !s->axisym && (s->tly.nt || s->tll.nt)) {
         const std::vector<std::pair<int, int>> nts{{128, 128}, {256, 256},  {256, 512},
                                                    {512, 512}, {256, 1024}, {512, 1024}};
-        const bool py = s->g.dim == 3 && s->axY.n >= 160, pl = s->axL.n >= 160;
-        for (const auto& pe : nts)
+        const bool ty = s->tly.nt != 0, tl = s->tll.nt != 0;
+        const bool py = ty && s->axY.n >= 160, pl = tl && s->axL.n >= 160;
+        std::set<std::pair<int, int>> timed;
+        for (const auto& pe : nts) {
+          if (!timed.insert({ty ? pe.first : 0, tl ? pe.second : 0}).second) continue;
           for (int a = 0; a <= (py ? 1 : 0); ++a)
             for (int b = 0; b <= (pl ? 1 : 0); ++b) {
               TuneCfg c = best;
-              c.pencil_y = pe.first;
-              c.pencil_last = pe.second;
+              if (ty) c.pencil_y = pe.first;
+              if (tl) c.pencil_last = pe.second;
               c.plan_y = a;
               c.plan_last = b;
               c.narrow = 0;
               trial(c);
             }
+        }
       }
       if (s->g.kxm)
         for (int pn : (s->g.Ny * s->g.Nz < 16384 ? std::vector<int>{256, 512, 1024} : std::vector<int>{512, 1024})) {

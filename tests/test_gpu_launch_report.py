@@ -1,4 +1,5 @@
-"""kw_sim_launch_config names the workgroup sizes and radix plans that run."""
+"""kw_sim_launch_config names the workgroup sizes and radix plans that run, and the
+autotuner times each launch shape once."""
 
 import pytest
 
@@ -45,3 +46,16 @@ def test_generic_kernels_report_zero(kw, monkeypatch):
         monkeypatch.setenv(k, "0")
     c = config(kw, cases.case_3d(N=(54, 45, 48), Nt=4, pml=4, source="p"))
     assert (c["row_nt"], c["ypass_nt"], c["last_nt"], c["ypass_plan"], c["last_plan"]) == (0, 0, 0, 0, 0)
+
+
+def test_autotuner_times_each_shape_once(kw):
+    """A tuned y axis beside a last axis with one instantiation: the base, three row
+    workgroup sizes, three row targets, and three y-pass sizes.  The first step of a
+    trial and the timed ones launch one density kernel each."""
+    f = cases.case_3d(N=(64, 48, 35), Nt=12, pml=4, source="p")
+    with kw.Simulation(f, record=("p",)) as sim:
+        sim.set_profiling(True)
+        sim.autotune(trial_steps=3)
+        launches = sim.profile()["x_density"][1]
+    print(f"[gpu launch report] 64x48x35: {launches} density launches", flush=True)
+    assert launches == (1 + 3 + 3 + 3) * 4
