@@ -64,7 +64,9 @@ def kernel_bytes(f: dict, kind: str) -> float:
     Counts each distinct array the kernel must read or write once: real
     fields 4 B/point, X-domain half spectra (Nx/2+1)*Ny*Nz*8 B, spectral
     tables 4 B per half-spectrum point; scalars and 1-D vectors 0.  The
-    spectral passes are averaged over one step's launches of that kind.
+    spectral passes are averaged over one step's launches of that kind; on
+    row-major 3-D grids the gradient's x and y outputs are one field between
+    the last axis and the y pass.
     """
     Nx, Ny, Nz = _dims(f)
     N = Nx * Ny * Nz
@@ -84,13 +86,14 @@ def kernel_bytes(f: dict, kind: str) -> float:
         fields = 1 + (1 if het("c0") else 0) + (2 if (het("c0") or het("alpha_coeff")) else 0)
         return 2 * spec + fields * fld + spec
     if kind in ("last_axis", "yz_plane"):  # in + out spectra + tables, averaged over the step's launches
-        # gradient 1->dim (+kappa), divergence dim->dim (+kappa), absorption 2->2 (+nabla1, nabla2)
-        launches = [(1, dim, 1), (dim, dim, 1)] + ([(2, 2, 2)] if absorbing == 1 else [])
+        # gradient 1->dim (+kappa; last axis of 3-D grids 1->2), divergence dim->dim (+kappa),
+        # absorption 2->2 (+nabla1, nabla2)
+        launches = [(1, 2 if kind == "last_axis" else dim, 1), (dim, dim, 1)] + ([(2, 2, 2)] if absorbing == 1 else [])
         return sum((i + o) * spec + t * tab for i, o, t in launches) / len(launches)
-    if kind == "y_pass":        # read + write of the fields of each launch: the inputs and the
-        # outputs of each spectral operator (gradient 1, dim; divergence dim, dim; absorption 2, 2)
-        nf = [1, dim, dim, dim] + ([2, 2] if absorbing == 1 else [])
-        return sum(2 * n * spec for n in nf) / len(nf)
+    if kind == "y_pass":        # fields read + written by each launch: the inputs and the outputs of
+        # each spectral operator (gradient 1 + 1, then 2 read and 3 written; divergence; absorption)
+        nf = [1 + 1, 2 + 3, 3 + 3, 3 + 3] + ([2 + 2, 2 + 2] if absorbing == 1 else [])
+        return sum(n * spec for n in nf) / len(nf)
     return 0.0
 
 
