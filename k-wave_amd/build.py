@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import concurrent.futures
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -39,10 +40,12 @@ HIP_FLAGS = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument",
 ]
 
-SOLVER_SOURCES = (["kw_kernels.hip", "kw_sim.cpp", "kw_server.cpp", "kw_plane.hip", "kw_axisym.hip", "kw_noalloc.hip"]
-                  + [f"kw_pencil_nt{n}.hip" for n in (128, 256, 512, 1024)]
-                  + [f"kw_xrow_nt{n}.hip" for n in (64, 128, 256)] + [f"kw_len_{i}.hip" for i in range(8)]
+# (the units that compile longest first)
+SOLVER_SOURCES = ([f"kw_xrow_nt{n}.hip" for n in (64, 128, 256)]
+                  + [f"kw_pencil_nt{n}.hip" for n in (128, 256, 512, 1024)] + ["kw_plane.hip"]
+                  + ["kw_kernels.hip", "kw_sim.cpp", "kw_server.cpp", "kw_axisym.hip", "kw_noalloc.hip"]
                   + ["kw_pencil_narrow.hip", "kw_axisym_fast.hip"])
+LEN_SOURCE = "kw_len.hip"  # compiled once per length of KW_LEN_SIZES
 IO_SOURCES = ["kw_io.cpp"]
 
 
@@ -58,8 +61,21 @@ def _run(cmd, verbose):
         print(out, flush=True)
 
 
-def _obj(src):
-    return os.path.join(LIB, "obj", os.path.splitext(src)[0] + ".o")
+def _obj(src, tag=""):
+    return os.path.join(LIB, "obj", os.path.splitext(src)[0] + tag + ".o")
+
+
+def len_sizes() -> list:
+    """The lengths of KW_LEN_SIZES (kw_kernels.hpp)."""
+    text = open(os.path.join(CSRC, "kw_kernels.hpp")).read()
+    macro = re.search(r"#define KW_LEN_SIZES\(X\)((?:.*\\\n)*.*)\n", text).group(1)
+    return [int(n) for n in re.findall(r"X\((\d+)\)", macro)]
+
+
+def solver_units() -> list:
+    """(source, object, extra flags) of each translation unit of the solver."""
+    return ([(s, _obj(s), []) for s in SOLVER_SOURCES]
+            + [(LEN_SOURCE, _obj(LEN_SOURCE, f"_{n}"), [f"-DKW_LENGTH={n}"]) for n in reversed(len_sizes())])
 
 
 def hdf5_available() -> bool:
@@ -72,11 +88,12 @@ def build(verbose: bool = False, with_io: bool = True) -> dict:
     os.makedirs(os.path.join(LIB, "obj"), exist_ok=True)
     os.makedirs(BIN, exist_ok=True)
     inc = [f"-I{INCLUDE}", f"-I{CSRC}"]
-    objs = [_obj(src) for src in SOLVER_SOURCES]
+    units = solver_units()
+    objs = [o for _, o, _ in units]
     # translation units compile in parallel (the length-specialised kernels dominate)
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(len(objs), os.cpu_count() or 1)) as ex:
-        futs = [ex.submit(_run, [HIPCC, *HIP_FLAGS, *inc, "-c", os.path.join(CSRC, src), "-o", o], verbose)
-                for src, o in zip(SOLVER_SOURCES, objs)]
+        futs = [ex.submit(_run, [HIPCC, *HIP_FLAGS, *extra, *inc, "-c", os.path.join(CSRC, src), "-o", o], verbose)
+                for src, o, extra in units]
         for fu in futs:
             fu.result()
     solver = os.path.join(LIB, "libkwave_hip.so")

@@ -772,20 +772,19 @@ bool fast_length(int n) {
   }
 }
 
-const LenKernels* len_kernels_0(int n);
-const LenKernels* len_kernels_1(int n);
-const LenKernels* len_kernels_2(int n);
-const LenKernels* len_kernels_3(int n);
-const LenKernels* len_kernels_4(int n);
-const LenKernels* len_kernels_5(int n);
-const LenKernels* len_kernels_6(int n);
-const LenKernels* len_kernels_7(int n);
+#define KW_CASE(n) const LenKernels* len_kernels_##n();
+KW_LEN_SIZES(KW_CASE)
+#undef KW_CASE
 const LenKernels* len_kernels(int n) {
-  using Find = const LenKernels* (*)(int);
-  for (Find f : {len_kernels_0, len_kernels_1, len_kernels_2, len_kernels_3,
-                 len_kernels_4, len_kernels_5, len_kernels_6, len_kernels_7})
-    if (const LenKernels* k = f(n)) return k;
-  return nullptr;
+  switch (n) {
+#define KW_CASE(n) \
+  case n:          \
+    return len_kernels_##n();
+    KW_LEN_SIZES(KW_CASE)
+#undef KW_CASE
+    default:
+      return nullptr;
+  }
 }
 
 // dispatch to the length-specialised kernels instantiated for `nt` threads

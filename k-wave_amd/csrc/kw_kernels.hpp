@@ -362,7 +362,7 @@ struct BatchClock {
 struct AsTables;
 using RadialFn = void (*)(hipStream_t, const Grid&, const AsTables&, const LastArgs&, float scale);
 
-// Launchers of the kernels of one axis length outside KW_FAST_SIZES (kw_len.inc).
+// Launchers of the kernels of one axis length outside KW_FAST_SIZES (kw_len.hip).
 struct LenKernels {
   void (*xvel)(hipStream_t, const Grid&, const float2* tw, const Medium&, float2* const* G, float* const* u,
                const Src*, const Sens*, int init);
@@ -400,11 +400,21 @@ struct TileLaunch {
   const LenKernels* len = nullptr;  // with nt 0: the length's kernels (nullptr = generic only)
 };
 
-// Axis lengths with compiled length-specialised kernels (kw_pencil_nt*.hip,
-// kw_xrow_nt*.hip, instantiated for 64-, 128- and 256-thread workgroups; the
-// pencils also for 512).
+// Tuned axis lengths: x rows in workgroups of 64, 128 and 256 threads
+// (kw_xrow_nt*.hip), pencils of 128 to 1024 (kw_pencil_nt*.hip).
 #define KW_FAST_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(384) X(512) X(768)
 bool fast_length(int n);
+// The other lengths of 32 .. 1024 without a prime factor above 7: kw_len.hip, one
+// module each, found by len_kernels().
+#define KW_LEN_SIZES(X) \
+  X(35) X(36) X(40) X(42) X(45) X(49) X(50) X(54) X(56) X(60) X(63) X(70) X(72) X(75) X(80) X(81) X(84) X(90) \
+  X(98) X(100) X(105) X(108) X(112) X(120) X(125) X(126) X(135) X(140) X(144) X(147) X(150) X(162) X(168) \
+  X(175) X(180) X(189) X(196) X(200) X(210) X(216) X(224) X(225) X(240) X(243) X(245) X(250) X(252) X(270) \
+  X(280) X(288) X(294) X(300) X(315) X(320) X(324) X(336) X(343) X(350) X(360) X(375) X(378) X(392) X(400) \
+  X(405) X(420) X(432) X(441) X(448) X(450) X(480) X(486) X(490) X(500) X(504) X(525) X(540) X(560) X(567) \
+  X(576) X(588) X(600) X(625) X(630) X(640) X(648) X(672) X(675) X(686) X(700) X(720) X(729) X(735) X(750) \
+  X(756) X(784) X(800) X(810) X(840) X(864) X(875) X(882) X(896) X(900) X(945) X(960) X(972) X(980) X(1000) \
+  X(1008) X(1024)
 constexpr bool tuned_length(int n) {
 #define KW_CASE(m) \
   if (n == m) return true;
