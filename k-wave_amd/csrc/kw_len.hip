@@ -23,9 +23,16 @@
 
 namespace kw {
 
-// pencil workgroup sizes, as for the tuned lengths: last axis 512 threads from
-// 384 points up and 1024, whose tile is the CU's, from 512 up (so is the y pass's
-// where no two workgroups of 512 with their tables fit a CU)
+// Pencil workgroup sizes by the rules of the tuned lengths.  Last axis: 512 threads
+// from 384 points up and 1024, whose tile is the CU's, from 512 up; us a launch at
+// 128x128xN with 256 / 512 / 1024 threads: 189 points 21.7 / 19.5 / 24.8, 252 30.5 /
+// 29.4 / 26.3, 350 39.2 / 39.9 / 40.3, 448 53.7 / 42.7 / 42.2, 525 75.9 / 63.8 / 69.3,
+// 640 97 / 85 / 76, 1000 284 / 182 / 120; below 512 some lengths would run up to a
+// third faster with more threads (270 38.2 / 26.2 / 30.4, 392 68.8 / 50.8 / 39.4).
+// Y pass: 512 from 256 up, and 1024 where no two workgroups of 512 with their
+// tables fit a CU; at 128xNx128: 189 15.8 / 14.8 / 16.9, 252 21.1 / 18.6 / 19.4, 270
+// 21.4 / 18.4 / 20.7, 392 34.6 / 26.6 / 27.1, 525 51.7 / 41.6 / 37.3, 640 61.5 / 53.0 /
+// 48.7, 1000 105 / 79 / 80.
 constexpr int len_last_nt(int n) { return n >= 512 ? 1024 : n >= 384 ? 512 : 256; }
 template <int N>
 constexpr int len_y_nt() {
